@@ -236,3 +236,45 @@ def test_q4_gemm_prefill_projection_size(gpu):
     mag = (x.float().abs() @ deq.abs().T).double()
     err = (y.double() - full).abs()
     assert bool((err <= 2e-5 * mag + 1e-5).all()), f"max err {err.max().item():.3e}"
+
+
+MANY_CASES = [
+    # M, N, K: rec_q4_gemm's kernels at the edges of their tiles and of their ranges
+    (9, 300, 256),        # few vectors, one row tile x 16 vectors per workgroup
+    (32, 2048, 4096),     # its largest grid (256 workgroups)
+    (33, 2040, 384),      # two row tiles x 16 vectors, a ragged last tile, three spans
+    (24, 5120, 128),      # two row tiles x 32 vectors, fewer spans than waves
+    (100, 2033, 2048),
+    (9, 8190, 128),       # streamed row tiles, 16 vectors, one span
+    (17, 8209, 1152),     # 32 vectors, nine spans: one wave with two
+    (32, 12288, 2048),
+    (200, 12288, 384),    # 64-vector tiles, two wave sets, 192 workgroups
+    (65, 24001, 128),     # a vector past the tile, one row past it, one group per set
+    (520, 8190, 256),     # one wave set, 288 workgroups
+    (1030, 4112, 640),
+]
+
+
+@pytest.mark.parametrize("case", MANY_CASES, ids=lambda c: f"M{c[0]}_N{c[1]}_K{c[2]}")
+def test_q4_many_rows_matches_oracle(gpu, case):
+    """More than 8 rows of x, strided: the first, last and some sampled output rows within
+    1e-5·(|x|·|W|ᵀ) of the float64 oracle (the module's bound), bf16 outputs the RNE of
+    the fp32 ones, and a vector of NaN and infinities leaves every other vector as it was."""
+    M, N, K = case
+    x, w, s, b = problem(M, N, K, seed=3 * M + N + K)
+    big = torch.zeros((M, K + 8), dtype=torch.bfloat16, device="cuda")
+    big[:, :K] = x
+    m = Q4Matrix(w, s, b)
+    y32 = q4_gemv(big[:, :K], m, out_dtype=torch.float32)
+    y16 = q4_gemv(x, m)
+    torch.cuda.synchronize()
+    rows = np.unique(np.r_[0:min(N, 70), max(0, N - 70):N, np.random.default_rng(N).choice(N, min(N, 60), replace=False)])
+    ref, mag = oracle_rows(x, w, s, b, rows)
+    check(y32[:, rows], ref, mag, f"case {case}")
+    assert torch.equal(y16.view(torch.int16), y32.to(torch.bfloat16).view(torch.int16)), "bf16 output is not RNE(fp32)"
+    bad = M // 2
+    x[bad, ::3] = float("inf")
+    x[bad, 1::3] = float("nan")
+    y = q4_gemv(x, m, out_dtype=torch.float32)
+    keep = [i for i in range(M) if i != bad]
+    assert torch.equal(y[keep], y32[keep]) and not bool(torch.isfinite(y[bad]).any())

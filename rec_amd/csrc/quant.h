@@ -242,4 +242,227 @@ __device__ __forceinline__ void append_v4_pair(const RowSrc& src, int b, int h, 
   codes[a1] = (uint8_t)(lo1 | (hi1 << 4));
 }
 
+// ---- whole blocks: one wavefront per 32-token block ----
+// Lane (kg, c) = (lane / 16, lane % 16) owns dims 8c .. 8c+7 of the eight
+// tokens 4kg .. 4kg+3 and 16+4kg .. 16+4kg+3, which are the block's positions
+// 8kg .. 8kg+7: a row's 16-byte runs load as one contiguous row per 16 lanes, a
+// quantization group lies in 16 (int8), 4 (uint4) or 8 (affine) adjacent lanes,
+// and every code it makes leaves in runs of 64 contiguous bytes per 8 or 16
+// lanes without an exchange between lanes.
+
+// a / b for several a of one b, in fewer instructions than the IEEE sequence.
+// y = RN(1/b).  q0 = RN(a y) is within 2 ulp of a/b, q1 = RN(q0 + (a - b q0) y)
+// within one, and q2 = RN(q1 + (a - b q1) y) is RN(a/b) (Markstein 1990: y
+// correctly rounded, q1 faithful, the residual exact in an fma) while nothing
+// overflows or turns subnormal, which the callers see to.
+//
+// EASY: a and b have at most 11 significant bits (fp16 or bf16 inputs, an fp16
+// step) and only the rounding of a/b to an integer matters.  A quotient that
+// is not half an odd integer is at least 2^-14 away from the next one that is
+// (a 2^k / b - m / 2 with 11-bit integers a, b), far beyond q1's error; one that
+// is comes out of the residual step exactly.  So one step with the hardware's
+// approximate reciprocal gives the same integer.
+template <bool EASY>
+struct Quotient {
+  float b, y;
+  __device__ __forceinline__ explicit Quotient(float b_) : b(b_), y(EASY ? __builtin_amdgcn_rcpf(b_) : 1.0f / b_) {}
+  __device__ __forceinline__ float operator()(float a) const {
+    float q = a * y;
+    q = fmaf(fmaf(-q, b, a), y, q);
+    if constexpr (!EASY) q = fmaf(fmaf(-q, b, a), y, q);
+    return q;
+  }
+};
+constexpr float QUOTIENT_MAX = 1e20f;  // magnitudes up to this keep every step above in range
+
+template <int CTRL>
+__device__ __forceinline__ float max_step(float x) { return fmaxf(x, dpp_f<CTRL>(x)); }
+template <int CTRL>
+__device__ __forceinline__ float min_step(float x) { return fminf(x, dpp_f<CTRL>(x)); }
+
+// The codes of a lane's eight values of one token in the format of `BITS`,
+// with the group's scale and zero-point / bias bits: the arithmetic of
+// quantize_i8_pair, quantize_u4_pair and quantize_affine_pair.
+template <int BITS, bool EASY>
+__device__ __forceinline__ void quantize_eight(const float (&x)[8], int (&q)[8], uint16_t& sbits, uint16_t& zbits) {
+  zbits = 0;
+  if constexpr (BITS == 8) {
+    float amax = fabsf(x[0]);
+#pragma unroll
+    for (int j = 1; j < 8; ++j) amax = fmaxf(amax, fabsf(x[j]));
+    amax = row16_max(amax);
+    sbits = half_bits_saturate(amax / 127.0f);
+    const float s = half_bits_to_float(sbits);
+    if (__any(!(amax <= QUOTIENT_MAX))) {  // (wave-uniform; infinities, NaN rows)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) q[j] = s != 0.0f ? (int)fminf(fmaxf(__builtin_rintf(x[j] / s), -127.0f), 127.0f) : 0;
+    } else {
+      const Quotient<EASY> d(s != 0.0f ? s : 1.0f);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) q[j] = s != 0.0f ? (int)fminf(fmaxf(__builtin_rintf(d(x[j])), -127.0f), 127.0f) : 0;
+    }
+  } else if constexpr (BITS == 4) {
+    float mn = x[0], mx = x[0];
+#pragma unroll
+    for (int j = 1; j < 8; ++j) {
+      mn = fminf(mn, x[j]);
+      mx = fmaxf(mx, x[j]);
+    }
+    mn = min_step<DPP_XOR2>(min_step<DPP_XOR1>(mn));
+    mx = max_step<DPP_XOR2>(max_step<DPP_XOR1>(mx));
+    mn = fminf(mn, 0.0f);
+    mx = fmaxf(mx, 0.0f);
+    sbits = half_bits_saturate((mx - mn) / 15.0f);
+    const float s = half_bits_to_float(sbits);
+    float z = 0.0f;
+    if (__any(!(mx - mn <= QUOTIENT_MAX))) {
+      if (s != 0.0f) z = fminf(fmaxf(__builtin_rintf(-mn / s), 0.0f), 15.0f) + 0.0f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) q[j] = s != 0.0f ? (int)fminf(fmaxf(__builtin_rintf(x[j] / s) + z, 0.0f), 15.0f) : 0;
+    } else {
+      const Quotient<EASY> d(s != 0.0f ? s : 1.0f);
+      z = s != 0.0f ? fminf(fmaxf(__builtin_rintf(d(-mn)), 0.0f), 15.0f) + 0.0f : 0.0f;  // +0, never -0
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        q[j] = s != 0.0f ? (int)fminf(fmaxf(__builtin_rintf(d(x[j])) + z, 0.0f), 15.0f) : 0;
+    }
+    zbits = float_to_half_bits(z);
+  } else {
+    constexpr float n_bins = is_a8(BITS) ? 255.0f : 15.0f;
+    float mn = x[0], mx = x[0];
+#pragma unroll
+    for (int j = 1; j < 8; ++j) {
+      mn = fminf(mn, x[j]);
+      mx = fmaxf(mx, x[j]);
+    }
+    mn = min_step<DPP_HALF_MIRROR>(min_step<DPP_XOR2>(min_step<DPP_XOR1>(mn)));
+    mx = max_step<DPP_HALF_MIRROR>(max_step<DPP_XOR2>(max_step<DPP_XOR1>(mx)));
+    mx = fmaxf(mx, 0.0f);
+    float scale = fmaxf((mx - mn) / n_bins, 1e-7f);
+    const bool side = fabsf(mn) > fabsf(mx);
+    scale = side ? scale : -scale;
+    const float edge = side ? mn : mx;
+    const float qe = __builtin_roundf(edge / scale);
+    const bool at_zero = qe == 0.0f;
+    scale = at_zero ? scale : edge / qe;
+    const float bias = at_zero ? 0.0f : edge;
+    if (__any(!(mx - mn <= QUOTIENT_MAX))) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) q[j] = (int)fminf(fmaxf(__builtin_roundf((x[j] - bias) / scale), 0.0f), n_bins);
+    } else {
+      const Quotient<false> d(scale);  // at least about 1e-7 in magnitude, 24 bits
+#pragma unroll
+      for (int j = 0; j < 8; ++j) q[j] = (int)fminf(fmaxf(__builtin_roundf(d(x[j] - bias)), 0.0f), n_bins);
+    }
+    sbits = meta_f16(BITS) ? float_to_half_bits(scale) : float_to_bf16_bits(scale);
+    zbits = meta_f16(BITS) ? float_to_half_bits(bias) : float_to_bf16_bits(bias);
+  }
+}
+
+// Eight consecutive elements of a row, as loaded.
+template <bool F32>
+struct Eight {
+  v4i w[F32 ? 2 : 1];
+  __device__ __forceinline__ void load(const RowSrc& s, int64_t i) {
+    if constexpr (F32) {
+      w[0] = *(const v4i*)((const float*)s.p + i);
+      w[1] = *(const v4i*)((const float*)s.p + i + 4);
+    } else {
+      w[0] = *(const v4i*)((const uint16_t*)s.p + i);
+    }
+  }
+  __device__ __forceinline__ void values(int dtype, float (&x)[8]) const {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if constexpr (F32) {
+        const int u = w[j >> 2][j & 3];
+        x[j] = __builtin_bit_cast(float, u);
+      } else {
+        const uint32_t u = (uint32_t)w[0][j >> 1];
+        if (dtype == DT_F16) x[j] = half_bits_to_float((j & 1) ? u >> 16 : u & 0xffffu);
+        else x[j] = __builtin_bit_cast(float, (j & 1) ? u & 0xffff0000u : u << 16);
+      }
+    }
+  }
+};
+
+// Quantize tokens t_src .. t_src + 31 of row (b, h) of `src` into the 32-token
+// block at cache position `pos` (a multiple of 32).  IS_V: the V layouts.
+template <int BITS, bool IS_V, bool F32>
+__device__ __forceinline__ void append_block(const RowSrc& src, int b, int h, int t_src, void* codes, uint16_t* scales,
+                                             uint16_t* zeros, int64_t bh, int64_t cap, int64_t pos, int lane) {
+  const int kg = lane >> 4, c = lane & 15;
+  const int64_t base = row_base(src, b, h, t_src) + 8 * c;
+  Eight<F32> in[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) in[e].load(src, base + (int64_t)((e >> 2) * 16 + 4 * kg + (e & 3)) * src.st);
+  uint16_t sb[8], zb[8];  // by position e
+  uint32_t v[8][2];       // V codes of dim j: bytes (int8) or nibbles (4-bit) by position
+  constexpr bool BYTE = BITS == 8 || is_a8(BITS);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    float x[8];
+    int q[8];
+    in[e].values(src.dtype, x);
+    quantize_eight<BITS, !F32>(x, q, sb[e], zb[e]);
+    if constexpr (!IS_V) {
+      const int64_t t = pos + (e >> 2) * 16 + 4 * kg + (e & 3);
+      if constexpr (BYTE) {
+        v2i o;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          o[i] = (q[4 * i] & 0xff) | ((q[4 * i + 1] & 0xff) << 8) | ((q[4 * i + 2] & 0xff) << 16) | (q[4 * i + 3] << 24);
+        *(v2i*)((uint8_t*)codes + k8_off(bh, cap, t, 8 * c)) = o;
+      } else {
+        uint32_t o = 0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) o |= (uint32_t)q[j] << (4 * j);
+        *(uint32_t*)((uint8_t*)codes + k4_off(bh, cap, t, 8 * c)) = o;
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        if constexpr (BYTE) {
+          const uint32_t o = (uint32_t)(q[j] & 0xff) << (8 * (e & 3));
+          v[j][e >> 2] = (e & 3) ? v[j][e >> 2] | o : o;
+        } else {
+          const uint32_t o = (uint32_t)q[j] << (4 * e);
+          v[j][0] = e ? v[j][0] | o : o;
+        }
+      }
+    }
+  }
+  if constexpr (IS_V) {  // token 4kg is position 8kg of the block
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if constexpr (BYTE)
+        *(v2i*)((uint8_t*)codes + v8_off(bh, cap, pos + 4 * kg, 8 * c + j)) = (v2i){(int)v[j][0], (int)v[j][1]};
+      else
+        *(uint32_t*)((uint8_t*)codes + v4_off(bh, cap, pos + 4 * kg, 8 * c + j)) = v[j][0];
+    }
+  }
+  // one lane per group stores the eight positions' scales: int8 in order, the
+  // others in slot order (s4_slot: positions 0 4 1 5 2 6 3 7)
+  constexpr int GROUP_LANES = BITS == 8 ? 16 : (is_affine(BITS) ? 8 : 4);
+  if (c % GROUP_LANES == 0) {
+    const int g = c / GROUP_LANES;
+    v4i so, zo;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int lo = BITS == 8 ? 2 * i : i, hi = BITS == 8 ? 2 * i + 1 : i + 4;
+      so[i] = (int)(sb[lo] | ((uint32_t)sb[hi] << 16));
+      zo[i] = (int)(zb[lo] | ((uint32_t)zb[hi] << 16));
+    }
+    if constexpr (BITS == 8) {
+      *(v4i*)(scales + s8_off(bh, cap, pos + 4 * kg)) = so;
+    } else if constexpr (is_affine(BITS)) {
+      *(v4i*)(scales + sa_off(bh, cap, pos + 4 * kg, 0, g)) = so;
+      *(v4i*)(scales + sa_off(bh, cap, pos + 4 * kg, 1, g)) = zo;
+    } else {
+      *(v4i*)(scales + s4_off(bh, cap, pos + 4 * kg, g)) = so;
+      *(v4i*)(zeros + s4_off(bh, cap, pos + 4 * kg, g)) = zo;
+    }
+  }
+}
+
 }  // namespace rec

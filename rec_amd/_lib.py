@@ -117,6 +117,20 @@ SIGNATURES["rec_q4_gemm"] = (_i, [_p, _i64, _i64, _p, _i64, _i, _p, _i, _i64, _p
 
 _lock = threading.Lock()
 _lib = None
+_host = None
+
+
+def host():
+    """The module ``rec_amd/_host.so`` (csrc/host.cpp): the small calls' host path."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise RuntimeError(f"rec_amd host module not built or not loadable ({e}); run `python -m rec_amd.build`") from e
+        _host = module
+    return _host
 
 
 class RecError(RuntimeError):

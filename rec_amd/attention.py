@@ -615,6 +615,39 @@ def scaled_dot_product_attention(queries, keys, values, scale, mask=None, sinks=
     return _finish(out, want)
 
 
+def _decode_step(queries, keys, values, cache, scale, sinks):
+    """A decode step in its plain form (no mask, result in the query dtype, a
+    cache with room, a workspace that an earlier call made) through the native
+    host path, or None: :func:`attend` then takes the general path, which also
+    raises what there is to raise."""
+    dev = queries.get_device()
+    stream = torch._C._cuda_getCurrentRawStream(dev)
+    ws = _workspaces.get((dev, stream))
+    if ws is None:
+        return None
+    if isinstance(cache, QuantizedKVCache):
+        T = cache.offset + 1
+        if not cache._usable or cache.keys is None or T > cache.capacity \
+                or (cache.max_tokens is not None and T > cache.max_tokens):
+            return None
+        out = _lib.host().decode_quantized(
+            queries, keys, values, *cache.keys, cache.key_bits, *cache.values, cache.value_bits, cache.affine, sinks,
+            scale, T, cache.capacity, ws, stream)
+    elif isinstance(cache, FixedSlidingKVCache):
+        try:
+            sk = _sinks(sinks, queries.shape[1], queries.device, queries.dtype)
+        except ValueError:
+            return None
+        out = _lib.host().decode_ring(
+            queries, keys, values, cache.keys, cache.values, sk, scale, min(cache.offset + 1, cache.capacity),
+            cache.capacity, cache.offset % cache.capacity, ws, stream)
+    else:
+        return None
+    if out is not None:
+        cache.offset += 1
+    return out
+
+
 def attend(queries, keys, values, cache, scale, mask=None, sinks=None, *, out_dtype=None,
            splits=None, fused=True):
     """The cache + attention part of ``Attention.__call__`` (model.py:177-211).
@@ -635,6 +668,11 @@ def attend(queries, keys, values, cache, scale, mask=None, sinks=None, *, out_dt
     that pattern); a mask array on the GPU (never inspected: :func:`_mask_plan`)
     takes the append, then the masked attention.
     """
+    if mask is None and fused and out_dtype is None and splits is None and isinstance(queries, torch.Tensor) \
+            and queries.is_cuda and queries.dim() == 4 and queries.shape[2] == 1:
+        out = _decode_step(queries, keys, values, cache, scale, sinks)
+        if out is not None:
+            return out
     _check_query(queries)
     B, Hq, L, D = queries.shape
     qdt = queries.dtype

@@ -109,6 +109,17 @@ def q4_gemv(x: torch.Tensor, m: Q4Matrix, out_dtype=None) -> torch.Tensor:
     out_dtype = torch.bfloat16 if out_dtype is None else out_dtype
     if out_dtype not in (torch.bfloat16, torch.float32):
         raise ValueError(f"out_dtype must be bfloat16 or float32, got {out_dtype}")
+    # one GEMM over the packed matrix from 9 rows on, which reads the weights
+    # once: 2,048 x 4,096 at 9 / 24 rows 7.5 / 8.6 us against 11.5 / 21.8 in
+    # GEMV launches of 8.  A matrix of less than a tile, which no projection
+    # is, keeps the documented crossing gemm_min_rows (8 x 2,048 at 24 rows:
+    # 16.6 us in three launches, one would take 4.9)
+    gemm_rows = MAX_VECTORS + 1 if m.N >= 16 else gemm_min_rows(m.K)
+    if x.is_cuda:  # rows that need no copy: checked, allocated and launched natively
+        out = _lib.host().q4_matmul(x, m.packed, m.N, m.K, out_dtype is torch.float32, gemm_rows,
+                                    torch._C._cuda_getCurrentRawStream(x.get_device()))
+        if out is not None:
+            return out
     lead = x.shape[:-1]
     xs = x.reshape(-1, m.K)
     if xs.stride(-1) != 1 or xs.data_ptr() % 16 or (xs.shape[0] > 1 and xs.stride(0) % 8):
@@ -118,12 +129,7 @@ def q4_gemv(x: torch.Tensor, m: Q4Matrix, out_dtype=None) -> torch.Tensor:
     lib = _lib.load()
     stream = torch.cuda.current_stream(x.device).cuda_stream
     code = _lib.REC_F32 if out_dtype == torch.float32 else _lib.REC_BF16
-    if rows > MAX_VECTORS and (m.N >= 16 or rows >= gemm_min_rows(m.K)):
-        # one GEMM over the packed matrix, which reads the weights once: 2,048
-        # x 4,096 at 9 / 24 rows 7.5 / 8.6 us against 11.5 / 21.8 in GEMV
-        # launches of 8.  A matrix of less than a tile, which no projection
-        # is, keeps the documented crossing gemm_min_rows (8 x 2,048 at 24
-        # rows: 16.6 us in three launches, one would take 4.9)
+    if rows >= gemm_rows:  # x's group sums in a workspace first
         ws = torch.empty(lib.rec_q4_gemm_workspace_bytes(rows, m.K), dtype=torch.uint8, device=x.device)
         rc = lib.rec_q4_gemm(
             m.packed.data_ptr(), m.N, m.K, xs.data_ptr(), xs.stride(0), rows, out.data_ptr(), code, out.stride(0),

@@ -208,7 +208,8 @@ int rec_decode_merge(const float* sinks, int B, int Hq, int Hkv, int64_t T, int 
  * bias, causal and window must be 0 (the bias carries the whole mask) and the
  * chunk takes the tiled kernel.  Any cache format of rec_decode_attn (int8 or uint4
  * in any mix, or an affine pair): K/V tiles are dequantized into on-chip
- * memory, never to HBM — int8 codes exactly with the row scales applied to
+ * memory (or once into the workspace, see
+ * rec_prefill_quantized_workspace_bytes) — int8 codes exactly with the row scales applied to
  * scores and probabilities, 4-bit and affine values as x̂ rounded to the
  * query dtype, as the reference dequantizes before its attention.  A chunk
  * of at most 32 (query, head) rows per KV head (64 over a cache of 16,384
@@ -239,6 +240,14 @@ int rec_prefill_attn(const void* q, int q_dtype, int64_t q_sb, int64_t q_sh, int
  * Serves rec_prefill_attn and rec_prefill_bf16; no counterpart in the
  * reference, whose prefill is one library call. */
 size_t rec_prefill_workspace_bytes(int B, int Hq, int Hkv, int L, int splits);
+
+/* The workspace bytes with which rec_prefill_attn runs a chunk over a quantized
+ * cache of T tokens fastest: the above and, for a long chunk without a window
+ * or a bias, room for the cache's dequantized tiles (584 bytes per token and KV
+ * head, at most 1 GiB), which the launch then makes once for all its query
+ * blocks.  With the smaller workspace every query block dequantizes the tiles
+ * it reads itself; the results are the same. */
+size_t rec_prefill_quantized_workspace_bytes(int B, int Hq, int Hkv, int L, int64_t T, int splits);
 
 /*
  * bf16 KV cache (the reference's production format): K and V are (B, Hkv,

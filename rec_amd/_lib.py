@@ -71,6 +71,7 @@ SIGNATURES["rec_prefill_attn"] = (
      _p, _i64, _i64, _i64, _i64, _i64,  # bias, strides (b, kv head, group member, query), extent
      _i, _i, _i, _i, _i, _i64, _i64, _i, _p, _sz, _i, _p, _p],
 )
+SIGNATURES["rec_prefill_quantized_workspace_bytes"] = (_sz, [_i, _i, _i, _i, _i64, _i])
 SIGNATURES["rec_prefill_workspace_bytes"] = (_sz, [_i, _i, _i, _i, _i])
 
 SIGNATURES["rec_kv_write_bf16"] = (

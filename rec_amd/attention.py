@@ -212,7 +212,18 @@ def _prefill_launch(queries, keys: QuantizedKV, values: QuantizedKV, scale, sink
     dev = queries.device
     sk = _sinks(sinks, Hq, dev, sink_dtype)
     stream = torch.cuda.current_stream(dev).cuda_stream
-    ws = prefill_workspace(dev, B, Hq, keys.n_kv_heads, L, splits, stream)
+    ws = None
+    if window == 0 and bias is None:
+        # a long chunk's workspace holds the dequantized tiles as well (up to
+        # 1 GiB): allocated for the call and given back, not kept
+        full = lib.rec_prefill_quantized_workspace_bytes(B, Hq, keys.n_kv_heads, L, int(keys.length), splits)
+        if full > lib.rec_prefill_workspace_bytes(B, Hq, keys.n_kv_heads, L, splits):
+            try:
+                ws = torch.empty(full, dtype=torch.uint8, device=dev)
+            except torch.OutOfMemoryError:
+                pass  # the launch works without them
+    if ws is None:
+        ws = prefill_workspace(dev, B, Hq, keys.n_kv_heads, L, splits, stream)
     rc = lib.rec_prefill_attn(
         q.data_ptr(), _DTYPES[q.dtype], q.stride(0), q.stride(1), q.stride(2),
         keys.code, keys.codes.data_ptr(), keys.scales.data_ptr(), _ptr(keys.zeros),

@@ -544,7 +544,20 @@ int rec_prefill_attn(const void* q, int q_dtype, int64_t q_sb, int64_t q_sh, int
   a.causal = causal != 0;
   a.window = window;
   if ((e = plan_prefill_splits(a, splits, workspace, workspace_bytes))) return e;
+  // room behind the partials for the dequantized tiles: the workgroups then
+  // load those instead of dequantizing each tile themselves (same results)
+  const size_t img = window == 0 && !bias && workspace && aligned16(workspace) && !prefill_few_fits(a)
+                         ? prefill_image_bytes(B, Hkv, a.G, L, T) : 0;
+  const size_t parts = round256(prefill_ws_bytes(B, Hkv, (int64_t)a.nqb * a.block_rows, a.S));
+  if (img > 0 && workspace_bytes >= parts + img) a.img = (char*)workspace + parts;
   return launched(launch_prefill(a, (hipStream_t)stream), "prefill launch");
+}
+
+size_t rec_prefill_quantized_workspace_bytes(int B, int Hq, int Hkv, int L, int64_t T, int splits) {
+  const size_t parts = rec_prefill_workspace_bytes(B, Hq, Hkv, L, splits);
+  if (B < 1 || Hkv < 1 || L < 1 || Hq < Hkv || Hq % Hkv != 0 || T < L) return parts;
+  const size_t img = prefill_image_bytes(B, Hkv, Hq / Hkv, L, T);
+  return img > 0 ? round256(parts) + img : parts;
 }
 
 int rec_kv_dequant_bf16(int k_bits, const void* k_codes, const uint16_t* k_scales, const uint16_t* k_zeros, int v_bits,

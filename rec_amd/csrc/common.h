@@ -46,6 +46,7 @@ __host__ __device__ constexpr bool is_a4(int f) { return f == FMT_A4 || f == FMT
 __host__ __device__ constexpr bool is_affine(int f) { return is_a8(f) || is_a4(f); }
 __host__ __device__ constexpr bool meta_f16(int f) { return f == FMT_A8H || f == FMT_A4H; }
 constexpr int FMT_BF = 16;  // bf16 K/V tensors (the KVStorage cache), prefill only
+constexpr int FMT_IMG = 20;  // tiles a prefill launch dequantized to memory first (prefill_image_kernel)
 constexpr int GROUP_A = 64;
 constexpr int BLOCK_T = 32;      // tokens per cache block and per wave iteration
 constexpr int GROUP4 = 32;       // int4 group size along head_dim

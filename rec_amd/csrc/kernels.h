@@ -98,6 +98,7 @@ struct PrefillArgs {
   int S, nqb, block_rows;      // splits, query blocks of block_rows (query, head) rows
   int64_t split_lo, split_len;
   BiasArgs bias;               // additive score bias (a mask array), or none
+  char* img;                   // dequantized tiles [B*Hkv][ceil(T/128)][PREFILL_IMG_TILE], or null
   float* ws_acc;               // [B*Hkv][S][nqb][block_rows][128]
   float* ws_stat;              // [B*Hkv][S][nqb][block_rows] x (max, sum)
 };
@@ -116,6 +117,12 @@ struct PrefillPlan {
 // requested <= 0: automatic (splits only when the query blocks x KV heads x
 // batch grid is too small to fill the chip); else at most `requested`
 PrefillPlan prefill_plan(const PrefillArgs& a, int requested);
+// A chunk of many queries over a quantized cache (no window, no mask array)
+// dequantizes every tile once into the workspace, as the image its workgroups
+// then load straight into LDS: bytes of those images, 0 where the launch
+// dequantizes in its workgroups.
+constexpr int PREFILL_IMG_TILE = 2 * 128 * 144 * 2 + 2 * 128 * 4;
+size_t prefill_image_bytes(int B, int Hkv, int G, int L, int64_t T);
 // workspace bytes for S splits of head_rows (= nqb x block_rows) rows per KV
 // head (0 when S == 1); accumulators then statistics
 size_t prefill_ws_bytes(int B, int Hkv, int64_t head_rows, int S);

@@ -53,11 +53,22 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "dma.h"
 #include "kernels.h"
 
 namespace rec {
 
 constexpr int PF_ROWS = PREFILL_BLOCK_ROWS;  // (query, head) rows per workgroup: 16 tiles of 16
+// Query rows per KV head and keys from which the tiles are dequantized ahead
+// (12 query blocks share each image), and the most memory their images may
+// take.  bf16 queries, 32 q / 4 kv heads, dequantized in the workgroups → ahead,
+// images included, µs: 384 queries after 8,192 tokens int8 128.4 → 118.7,
+// uint4 142.5 → 118.6, affine 142.8 → 118.4; 1,500 after 32,768 int8 1,128 → 970,
+// uint4 1,288 → 974, affine 1,312 → 973; 2,048 after 65,536 int8 2,196 → 1,966.
+// Below the line the images cost what they save: 256 queries after 8,192 int8
+// 62.5 → 61.3, after 32,768 160.5 → 169.2; 1,500 after 2,048 168.6 → 169.2.
+constexpr int64_t PREFILL_IMG_ROWS = 12 * PREFILL_BLOCK_ROWS, PREFILL_IMG_KEYS = 4096;
+constexpr int64_t PREFILL_IMG_MAX = (int64_t)1 << 30;
 constexpr int PF_KROW = 144;  // LDS row pitch of K (elements): 128 + 16 pad
 
 // Tile geometry per cache format pair.
@@ -82,7 +93,7 @@ struct PfGeom {
   // int8/uint4 pair; the affine pair with the exact P·V); the bf16 cache's
   // transposed reads measured fastest issued at the P·V
   static constexpr int vpre(bool exact) {
-    return VTR ? 0 : ((KF == 8 && VF == 4) || (KF == 4 && VF == 8) || (exact && is_a8(KF))) ? 4 : 8;
+    return KF == FMT_IMG ? 8 : VTR ? 0 : ((KF == 8 && VF == 4) || (KF == 4 && VF == 8) || (exact && is_a8(KF))) ? 4 : 8;
   }
   // Scale bytes per 32-token block, per staged region: [K scales][K zeros][V scales][V zeros]
   // (int8: one fp16 per token; uint4: [4 groups][32 slots] fp16 scales, zero-points alike;
@@ -616,10 +627,21 @@ __global__ __launch_bounds__(512) void prefill_kernel(const PrefillArgs a) {
   typedef typename MT<BF16>::elem E;
   typedef typename MT<BF16>::vec V8;
   constexpr int KT = GEO::KT, U = GEO::U, VROW = GEO::VROW;
+  constexpr bool IMG = KF == FMT_IMG;
   __shared__ __attribute__((aligned(16))) E Kl[2][GEO::K_ELEMS];
   __shared__ __attribute__((aligned(16))) _Float16 Vl[2][GEO::V_ELEMS];
-  __shared__ __attribute__((aligned(16))) float KS[2][KT];
-  __shared__ __attribute__((aligned(16))) float VS[2][KT];
+  // the scales of K and V, both buffers (an image holds a tile's together)
+  __shared__ __attribute__((aligned(16))) float KSl[IMG ? 1 : 2][IMG ? 1 : KT];
+  __shared__ __attribute__((aligned(16))) float VSl[IMG ? 1 : 2][IMG ? 1 : KT];
+  __shared__ __attribute__((aligned(16))) float SCl[IMG ? 2 : 1][IMG ? 2 * KT : 1];
+  const auto KS = [&](int bf) -> float* {
+    if constexpr (IMG) return SCl[bf];
+    else return KSl[bf];
+  };
+  const auto VS = [&](int bf) -> float* {
+    if constexpr (IMG) return SCl[bf] + KT;
+    else return VSl[bf];
+  };
   __shared__ __attribute__((aligned(16))) char stage[GEO::STAGE > 0 ? GEO::STAGE : 16];
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -704,7 +726,24 @@ __global__ __launch_bounds__(512) void prefill_kernel(const PrefillArgs a) {
     if (GEO::STAGE > 0 && 8 * tid < GEO::STAGE) *(v2i*)(stage + 8 * tid) = R.sc;
   };
   const auto convert = [&](const TileRegs& R, int bf, auto phase) {
-    convert_tile<BF16, KF, VF, decltype(phase)::value>(R, Kl[bf], Vl[bf], KS[bf], VS[bf], stage, tid, a.q_mul);
+    convert_tile<BF16, KF, VF, decltype(phase)::value>(R, Kl[bf], Vl[bf], KS(bf), VS(bf), stage, tid, a.q_mul);
+  };
+  // IMG: the tile at t0 straight into buffer bf, 73 KB in 1 KB loads, wave w
+  // taking pieces w, w + 8, ...; dma_wait() and a barrier before it is read
+  const char* img = IMG ? a.img + bh * ((a.T + KT - 1) / KT) * PREFILL_IMG_TILE : nullptr;
+  const auto dma_tile = [&](int t0, int bf) {
+    if constexpr (IMG) {
+      const char* src = uniform_ptr(img + (int64_t)(t0 / KT) * PREFILL_IMG_TILE + 1024 * w);
+      constexpr int KP = GEO::K_ELEMS * 2 / 1024, VP = GEO::V_ELEMS * 2 / 1024;  // pieces of K, of V
+      static_assert(KP * 1024 == GEO::K_ELEMS * 2 && VP * 1024 == GEO::V_ELEMS * 2 && 1024 * (KP + VP + 1) == PREFILL_IMG_TILE);
+      const uint32_t kl = lds_address(Kl[bf]), vl = lds_address(Vl[bf]);
+#pragma unroll
+      for (int j = 0; j < (KP + VP) / 8; ++j) {
+        const int piece = w + 8 * j;
+        dma16(piece < KP ? kl + 1024 * piece : vl + 1024 * (piece - KP), src + 8192 * j, 16 * lane);
+      }
+      if (w == 0) dma16(lds_address(*KS(bf)), src + 1024 * (KP + VP), 16 * lane);
+    }
   };
   using P0 = std::integral_constant<int, 0>;
   using P1 = std::integral_constant<int, 1>;
@@ -733,14 +772,20 @@ __global__ __launch_bounds__(512) void prefill_kernel(const PrefillArgs a) {
     // flight.  Unconditional even for an empty range (lo >= t_end): every load
     // then fails its liveness test and reads nothing.
     TileRegs R;
-    load_tile<KF, VF>(R, a, b, h, bh, lo, tid, t_end);
-    stage_scales(R);
-    __syncthreads();
-    convert(R, 0, P0{});
-    convert(R, 0, P1{});
-    convert(R, 0, P2{});
-    __syncthreads();
-    if (lo + KT < t_end) load_tile<KF, VF>(R, a, b, h, bh, lo + KT, tid, t_end);
+    if constexpr (IMG) {
+      if (lo < t_end) dma_tile(lo, 0);
+      dma_wait();
+      __syncthreads();
+    } else {
+      load_tile<KF, VF>(R, a, b, h, bh, lo, tid, t_end);
+      stage_scales(R);
+      __syncthreads();
+      convert(R, 0, P0{});
+      convert(R, 0, P1{});
+      convert(R, 0, P2{});
+      __syncthreads();
+      if (lo + KT < t_end) load_tile<KF, VF>(R, a, b, h, bh, lo + KT, tid, t_end);
+    }
 
     // Software pipeline over 32-token units: the scores of unit u+1 are computed
     // on the matrix cores while the VALU runs the softmax of unit u.  A tile's
@@ -769,14 +814,28 @@ __global__ __launch_bounds__(512) void prefill_kernel(const PrefillArgs a) {
             // the unit before: this tile's unit u - 1, or the previous tile's last
             const int pb_ = u == 0 ? buf ^ 1 : buf, po = u == 0 ? KT - 32 : 32 * (u - 1);
             softmax_pv_unit<VROW, GEO::VTR, EXACT, NRT, GEO::vpre(EXACT), MM == 2>(
-                sc[(u + 1) & 1], Vl[pb_] + (GEO::VTR ? po * GEO::VPB : po), KS[pb_] + po, VS[pb_] + po, m_use, thr,
+                sc[(u + 1) & 1], Vl[pb_] + (GEO::VTR ? po * GEO::VPB : po), KS(pb_) + po, VS(pb_) + po, m_use, thr,
                 l_run, acc, pend_t, t_end, qabs, a.causal, window, needs_mask(pend_t), c, g, rb, brow);
           }
         }
         pend = live;
         pend_t = tu;
+        if constexpr (IMG) {
+          // every wave is past the unit that read the other buffer: the next
+          // tile has the other three units' time to arrive in it
+          if (u == 0 && more) {
+            __syncthreads();
+            dma_tile(t0 + KT, buf ^ 1);
+          }
+        }
       }
-      if (more) {
+      if constexpr (IMG) {
+        if (more) {
+          dma_wait();
+          __syncthreads();
+          buf ^= 1;
+        }
+      } else if (more) {
         // The next tile, whose bytes had this whole tile to arrive, into the
         // other buffer: its scale bytes to the staging area, then (once every
         // wave has finished the unit that read the other buffer) the
@@ -796,7 +855,7 @@ __global__ __launch_bounds__(512) void prefill_kernel(const PrefillArgs a) {
       // visited, and a tile has an even number of units, so its scores are in sc[1])
       if (pend)
         softmax_pv_unit<VROW, GEO::VTR, EXACT, NRT, GEO::vpre(EXACT), MM == 2>(
-            sc[1], Vl[buf] + GEO::vunit(U - 1), KS[buf] + KT - 32, VS[buf] + KT - 32, m_use, thr, l_run, acc,
+            sc[1], Vl[buf] + GEO::vunit(U - 1), KS(buf) + KT - 32, VS(buf) + KT - 32, m_use, thr, l_run, acc,
             pend_t, t_end, qabs, a.causal, window, needs_mask(pend_t), c, g, rb, brow);
 
       // the rows again, from an opaque copy of the lane's column: recomputed
@@ -851,14 +910,47 @@ __global__ __launch_bounds__(512) void prefill_kernel(const PrefillArgs a) {
   else scan(std::integral_constant<int, 0>{});
 }
 
+// One tile of every (KV head, batch row), dequantized once for all the query
+// blocks that read it: the LDS image of the scan above ([K rows][V rows][K
+// scales][V scales]), a workgroup per tile.
+//
+// A workgroup of the scan spent 17% of its time on its own conversion of every
+// tile, and a chunk of 2,048 queries has 64 query blocks converting the same
+// tiles.  Bound by memory: 35 KB read and 73 KB written per tile.
+template <bool BF16, int KF, int VF>
+__global__ __launch_bounds__(512) void prefill_image_kernel(const PrefillArgs a) {
+  typedef PfGeom<KF, VF> GEO;
+  constexpr int KT = GEO::KT, KB = GEO::K_ELEMS * 2, VB = GEO::V_ELEMS * 2;
+  __shared__ __attribute__((aligned(16))) char tile[PREFILL_IMG_TILE];
+  __shared__ __attribute__((aligned(16))) char stage[GEO::STAGE];
+  const int tid = threadIdx.x, h = blockIdx.y, b = blockIdx.z;
+  const int64_t bh = (int64_t)b * a.Hkv + h;
+  TileRegs R;
+  load_tile<KF, VF>(R, a, b, h, bh, (int)blockIdx.x * KT, tid, (int)a.T);
+  if (8 * tid < GEO::STAGE) *(v2i*)(stage + 8 * tid) = R.sc;
+  // (the pads of the rows too: every byte of the image is written)
+  for (int i = tid; i < PREFILL_IMG_TILE / 16; i += 512) *(v4i*)(tile + 16 * i) = (v4i){0, 0, 0, 0};
+  __syncthreads();
+  typename MT<BF16>::elem* K = (typename MT<BF16>::elem*)tile;
+  _Float16* V = (_Float16*)(tile + KB);
+  float* KS = (float*)(tile + KB + VB);
+  convert_tile<BF16, KF, VF, 0>(R, K, V, KS, KS + KT, stage, tid, a.q_mul);
+  convert_tile<BF16, KF, VF, 1>(R, K, V, KS, KS + KT, stage, tid, a.q_mul);
+  convert_tile<BF16, KF, VF, 2>(R, K, V, KS, KS + KT, stage, tid, a.q_mul);
+  __syncthreads();
+  char* out = a.img + (bh * gridDim.x + blockIdx.x) * PREFILL_IMG_TILE;
+  for (int i = tid; i < PREFILL_IMG_TILE / 16; i += 512) *(v4i*)(out + 16 * i) = *(const v4i*)(tile + 16 * i);
+}
+
 // Merge of the key splits (S > 1): one wavefront per (query, query head,
 // batch); lane k owns the statistics of split k, the weights go through LDS,
 // and lane l sums dims 2l, 2l + 1 over the splits.  The sink logit joins here.
-// NR rounds of 16 split loads (S <= 16 NR), all issued before the first is
-// used: one trip to memory, not one per round.
-template <int NR>
+// NL split loads (S <= NL), all issued before the first is used: one trip to
+// memory, and few loads past the last split (1,000 queries x 32 heads of two
+// splits: 18.9 us with 16 loads, 11.0 with two).
+template <int NL>
 __global__ __launch_bounds__(64) void prefill_merge_kernel(const PrefillArgs a) {
-  static_assert(16 * NR <= PREFILL_MAX_SPLITS && PREFILL_MAX_SPLITS <= 64, "one split per lane");
+  static_assert(NL <= PREFILL_MAX_SPLITS && PREFILL_MAX_SPLITS <= 64, "one split per lane");
   const int i = blockIdx.x, hq = blockIdx.y, b = blockIdx.z, lane = threadIdx.x;
   const int h = hq / a.G, p = i * a.G + (hq - h * a.G);  // the (query, head) row
   const int qb = p / a.block_rows, r = p - qb * a.block_rows;
@@ -872,9 +964,9 @@ __global__ __launch_bounds__(64) void prefill_merge_kernel(const PrefillArgs a) 
   const uint32_t step_b = (uint32_t)a.nqb * a.block_rows * HEAD_DIM * 4;  // bytes between consecutive splits' rows
   const uint32_t last_b = (uint32_t)(a.S - 1) * step_b;              // below 2^31 (prefill_plan)
   const __amdgpu_buffer_rsrc_t racc = make_rsrc(a.ws_acc + row(0) * HEAD_DIM, (int64_t)last_b + HEAD_DIM * 4);
-  v2f x[16 * NR];
+  v2f x[NL];
 #pragma unroll
-  for (int k = 0; k < 16 * NR; ++k)
+  for (int k = 0; k < NL; ++k)
     x[k] = __builtin_bit_cast(v2f, ld64<0>(racc, 8 * lane, (uint32_t)min(k, a.S - 1) * step_b));
   float m = NEG_INF, l = 0.f;
   if (lane < a.S) {
@@ -890,7 +982,7 @@ __global__ __launch_bounds__(64) void prefill_merge_kernel(const PrefillArgs a) 
   // split k's weight is lane k's f (0 past the last split), read as a scalar
   v2f acc = {0.f, 0.f};
 #pragma unroll
-  for (int k = 0; k < 16 * NR; ++k)
+  for (int k = 0; k < NL; ++k)
     acc += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, f), k)) * x[k];
   const float inv = z > 0.f ? 1.f / z : 1.f;
   store_out2(a.out, (((int64_t)b * a.Hq + hq) * a.L + i) * HEAD_DIM + 2 * lane, acc * inv, a.out_dtype);
@@ -977,6 +1069,12 @@ PrefillPlan prefill_plan(const PrefillArgs& a, int requested) {
   return p;
 }
 
+size_t prefill_image_bytes(int B, int Hkv, int G, int L, int64_t T) {
+  if ((int64_t)L * G < PREFILL_IMG_ROWS || T < PREFILL_IMG_KEYS) return 0;
+  const int64_t bytes = (T + 127) / 128 * B * Hkv * PREFILL_IMG_TILE;
+  return bytes <= PREFILL_IMG_MAX ? (size_t)bytes : 0;
+}
+
 size_t prefill_ws_bytes(int B, int Hkv, int64_t head_rows, int S) {
   if (S <= 1) return 0;
   const size_t rows = (size_t)B * Hkv * S * head_rows;
@@ -994,6 +1092,18 @@ static void launch_quantized(const PrefillArgs& a, dim3 grid, dim3 block, hipStr
   else hipLaunchKernelGGL((prefill_kernel<BF16, FMT_A8H, FMT_A4H, EXACT, MM>), grid, block, 0, stream, a);
 }
 
+template <bool BF16>
+static void launch_image(const PrefillArgs& a, hipStream_t stream) {
+  const dim3 grid((unsigned)((a.T + 127) / 128), a.Hkv, a.B), block(512);
+  const int kf = a.k_fmt, vf = a.v_fmt;
+  if (kf == 8 && vf == 8) hipLaunchKernelGGL((prefill_image_kernel<BF16, 8, 8>), grid, block, 0, stream, a);
+  else if (kf == 8 && vf == 4) hipLaunchKernelGGL((prefill_image_kernel<BF16, 8, 4>), grid, block, 0, stream, a);
+  else if (kf == 4 && vf == 8) hipLaunchKernelGGL((prefill_image_kernel<BF16, 4, 8>), grid, block, 0, stream, a);
+  else if (kf == 4 && vf == 4) hipLaunchKernelGGL((prefill_image_kernel<BF16, 4, 4>), grid, block, 0, stream, a);
+  else if (kf == FMT_A8) hipLaunchKernelGGL((prefill_image_kernel<BF16, FMT_A8, FMT_A4>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((prefill_image_kernel<BF16, FMT_A8H, FMT_A4H>), grid, block, 0, stream, a);
+}
+
 // The bf16 cache (ring windows) always takes the window at run time; the
 // quantized formats have a variant with it and one without.  A bias (mask
 // array) takes its own variants, always with the exact P·V: a mask may leave
@@ -1005,6 +1115,9 @@ static void launch_formats(const PrefillArgs& a, dim3 grid, dim3 block, hipStrea
     else launch_quantized<BF16, true, 2>(a, grid, block, stream);
   } else if (a.k_fmt == FMT_BF) {
     hipLaunchKernelGGL((prefill_kernel<BF16, FMT_BF, FMT_BF, EXACT, 1>), grid, block, 0, stream, a);
+  } else if (a.img != nullptr) {
+    launch_image<BF16>(a, stream);
+    hipLaunchKernelGGL((prefill_kernel<BF16, FMT_IMG, FMT_IMG, EXACT, 0>), grid, block, 0, stream, a);
   } else if (a.window > 0) {
     launch_quantized<BF16, EXACT, 1>(a, grid, block, stream);
   } else {
@@ -1037,10 +1150,13 @@ hipError_t launch_prefill(const PrefillArgs& a, hipStream_t stream) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const dim3 grid((unsigned)a.L, a.Hq, a.B), block(64);
-    if (a.S <= 16) hipLaunchKernelGGL(prefill_merge_kernel<1>, grid, block, 0, stream, a);
-    else if (a.S <= 32) hipLaunchKernelGGL(prefill_merge_kernel<2>, grid, block, 0, stream, a);
-    else if (a.S <= 48) hipLaunchKernelGGL(prefill_merge_kernel<3>, grid, block, 0, stream, a);
-    else hipLaunchKernelGGL(prefill_merge_kernel<4>, grid, block, 0, stream, a);
+    if (a.S <= 2) hipLaunchKernelGGL(prefill_merge_kernel<2>, grid, block, 0, stream, a);
+    else if (a.S <= 4) hipLaunchKernelGGL(prefill_merge_kernel<4>, grid, block, 0, stream, a);
+    else if (a.S <= 8) hipLaunchKernelGGL(prefill_merge_kernel<8>, grid, block, 0, stream, a);
+    else if (a.S <= 16) hipLaunchKernelGGL(prefill_merge_kernel<16>, grid, block, 0, stream, a);
+    else if (a.S <= 32) hipLaunchKernelGGL(prefill_merge_kernel<32>, grid, block, 0, stream, a);
+    else if (a.S <= 48) hipLaunchKernelGGL(prefill_merge_kernel<48>, grid, block, 0, stream, a);
+    else hipLaunchKernelGGL(prefill_merge_kernel<64>, grid, block, 0, stream, a);
   }
   return hipGetLastError();
 }

@@ -6,6 +6,7 @@
 // covers 32 consecutive elements of one group -- lane (r, kq) takes word
 // 4t + kq of row r, dword kq of record lane r + 16t -- so the two groups of a
 // span accumulate apart.
+#include "dma.h"
 #include "q4.h"
 
 namespace rec {
@@ -43,27 +44,6 @@ constexpr int GM_X = GM_VECS * 128;
 constexpr int GM_W = 4 * 512;  // per wave: four tiles' codes
 constexpr int GM_SC = 256;     // per wave: four tiles' scale blocks
 constexpr int GM_STAGE = GM_X + 4 * (GM_W + GM_SC) + GM_VECS * 4;
-
-// Direct loads into LDS: lane i's 16 (4) bytes at p + voff arrive at lds + 16 i
-// (4 i).  Not tracked by the compiler: dma_wait() before the barrier in front
-// of the first read.
-__device__ __forceinline__ void dma16(uint32_t lds, const char* p, uint32_t voff) {  // p the same in every lane
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(p) : "memory");
-}
-__device__ __forceinline__ void dma16(uint32_t lds, const uint8_t* p) {  // p the lane's own
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "memory");
-}
-__device__ __forceinline__ void dma4(uint32_t lds, const char* p, uint32_t voff) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(voff), "s"(p) : "memory");
-}
-__device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-
-// A pointer that is the same in every lane, for a scalar register pair.
-__device__ __forceinline__ const char* uniform_ptr(const void* p) {
-  const uint64_t u = (uint64_t)p;
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)u), hi = __builtin_amdgcn_readfirstlane((uint32_t)(u >> 32));
-  return (const char*)(((uint64_t)hi << 32) | lo);
-}
 
 // Workgroup: 256 rows against 64 vectors, KS groups of four waves.  A wave
 // owns 64 rows (four row tiles) against all 64 vectors, so an x operand read
@@ -145,7 +125,7 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 3 : 2) void q4_gemm_kernel(cons
     wg[j] = a.packed + min(tile0 + 2 * j + (lane >> 5), tiles - 1) * S * GV_REC + 16 * (lane & 31);
   // lanes 0-15: row group lane % 4 of tile lane / 4
   const uint8_t* cg = a.packed + min(tile0 + (lane >> 2 & 3), tiles - 1) * S * GV_REC + 1024 + 32 * (lane & 3);
-  const uint32_t sm0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)sm + half * 2 * GM_STAGE;
+  const uint32_t sm0 = lds_address(sm) + half * 2 * GM_STAGE;
   const auto load = [&](int buf, int g) {
     const uint32_t l0 = sm0 + buf * GM_STAGE;
     const int64_t rec = (int64_t)(g >> 1) * GV_REC;

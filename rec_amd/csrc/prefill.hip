@@ -8,7 +8,8 @@
 // model.py:122-125 (query i sits at position T-L+i) and the per-head sink
 // logit in the softmax denominator.  The reference dequantizes the cache to
 // the query dtype (model.py:194-195) and runs one SDPA; here every K/V tile is
-// dequantized into LDS on the way from HBM, never written back:
+// dequantized into LDS on the way from HBM (for long chunks once for all
+// query blocks, as images of the LDS tiles in the workspace):
 //   * int8 K/V: the codes enter the matrix products exactly (|q| <= 127) and
 //     the row scales are applied outside them, the K scale to the scores, the
 //     V scale folded into the probabilities before their rounding;
